@@ -86,47 +86,57 @@ __global__ __launch_bounds__(256) void reduce_stage2(const A* __restrict__ parti
     }
 }
 
-// The whole reduction of a short vector in one workgroup, without the second
-// launch. Bound by the latency of its loads, four per lane in flight; the line
-// lies where they take longer than a launch: a set of nine calls with three
-// reductions takes 27.6 us with two launches each, in one 20.2 up to 6,000
-// elements, 22.8 (FP64) and 24.9 (FP32) at 16,000, 32.8 and 39.4 at 32,000.
-constexpr size_t kReduceOneMax = 16384;
-template <typename T, typename A, typename R>
-__global__ __launch_bounds__(1024) void reduce_one(RedOp op, const T* __restrict__ x, const T* __restrict__ y,
-                                                   uint32_t n, R* __restrict__ result, bool take_sqrt)
-{
-    constexpr int U = 4;
-    __shared__ A scratch[16];
-    A acc = A(0);
-    for (uint32_t i0 = threadIdx.x; i0 < n; i0 += U * 1024) {
-        T xv[U], yv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const uint32_t i = i0 + u * 1024;
-            xv[u] = i < n ? x[i] : T(0);
-            yv[u] = (y != nullptr && i < n) ? y[i] : T(0);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (i0 + u * 1024 < n) acc += red_term<T, A>(op, xv[u], yv[u]);
-    }
-    acc = wave_sum(acc);
-    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    A sum = A(0);
-    for (int w = 0; w < 16; ++w) sum += scratch[w];
-    if (take_sqrt) sum = static_cast<A>(sqrt(static_cast<double>(sum)));
-    *result = static_cast<R>(sum);
-}
-
 uint32_t reduce_blocks(size_t n)
 {
     size_t g = (n + 2047) / 2048;  // >= 8 elements per lane
     if (g < 1) g = 1;
     if (g > static_cast<size_t>(kReducePartialsMax)) g = kReducePartialsMax;
     return static_cast<uint32_t>(g);
+}
+
+// The whole reduction of a short vector in one workgroup, without the second
+// launch: the lanes of the (at most eight) workgroups of reduce_stage1 are this
+// one's, two per lane, and every sum is formed in the order of the two launches, so
+// the results are the same bits. (One chain of n / 1024 elements per lane and the
+// waves' sums one after the other instead: FP64 errors 1.1 to 1.6 times as large.)
+// Bound by the latency of its loads, all of a lane in flight at once; the line lies
+// at eight groups: a set of six FP64 calls, three of them reductions, takes 23.5 us
+// up to 6,000 elements, 24.7 at 16,384, and 33.3 from there on with two launches each.
+constexpr size_t kReduceOneMax = 16384;
+template <typename T, typename A, typename R>
+__global__ __launch_bounds__(1024) void reduce_one(RedOp op, const T* __restrict__ x, const T* __restrict__ y,
+                                                   uint32_t n, uint32_t g, R* __restrict__ result, bool take_sqrt)
+{
+    constexpr uint32_t kBlocks = kReduceOneMax / 2048, kChain = 8;  // elements of a lane of reduce_stage1 at most
+    __shared__ A scratch[kBlocks][4];
+    const uint32_t wave = (threadIdx.x >> 6) & 3, lane = threadIdx.x & 63;
+#pragma unroll
+    for (uint32_t q = 0; q < kBlocks / 4; ++q) {
+        const uint32_t block = 4 * q + (threadIdx.x >> 8);
+        const uint32_t first = block * 256 + (threadIdx.x & 255);
+        T xv[kChain], yv[kChain];
+#pragma unroll
+        for (uint32_t u = 0; u < kChain; ++u) {
+            const uint32_t i = first + u * g * 256;
+            const bool in = block < g && i < n;
+            xv[u] = in ? x[i] : T(0);
+            yv[u] = (y != nullptr && in) ? y[i] : T(0);
+        }
+        A acc = A(0);
+#pragma unroll
+        for (uint32_t u = 0; u < kChain; ++u)
+            if (block < g && first + u * g * 256 < n) acc += red_term<T, A>(op, xv[u], yv[u]);
+        acc = wave_sum(acc);
+        if (lane == 0) scratch[block][wave] = acc;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    A sum = A(0);
+    if (lane < g) sum = ((scratch[lane][0] + scratch[lane][1]) + scratch[lane][2]) + scratch[lane][3];
+    sum = wave_sum(sum);
+    if (lane != 0) return;
+    if (take_sqrt) sum = static_cast<A>(sqrt(static_cast<double>(sum)));
+    *result = static_cast<R>(sum);
 }
 
 enum class Ew { Add, Sub, Mul, Div };
@@ -359,13 +369,13 @@ clsparseStatus launch_reduce(RedOp op, const T* x, const T* y, size_t n, R* resu
                              bool sqrt_result, double* partials_buf, hipStream_t stream)
 {
     using A = typename AccOf<T>::type;
+    const uint32_t g = reduce_blocks(n);
     if (n <= kReduceOneMax) {
         hipLaunchKernelGGL((reduce_one<T, A, R>), dim3(1), dim3(1024), 0, stream, op, x, y, static_cast<uint32_t>(n),
-                           result, sqrt_result);
+                           g, result, sqrt_result);
         CLS_HIP_TRY(hipGetLastError());
         return clsparseSuccess;
     }
-    const uint32_t g = reduce_blocks(n);
     A* partials = reinterpret_cast<A*>(partials_buf);
     if (y == nullptr)
         hipLaunchKernelGGL((reduce_stage1<T, A, 4>), dim3(g), dim3(256), 0, stream, op, x, y, n, partials);
