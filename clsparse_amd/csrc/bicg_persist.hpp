@@ -1,42 +1,11 @@
-// Device state of one BiCGStab solve, and the persistent iteration as the
-// solver calls it (kernel in bicg_persist_kernel.hpp, one source per precision).
+// The persistent BiCGStab iteration as the solver calls it (kernel in
+// bicg_persist_kernel.hpp, one source per precision).
 #pragma once
 
+#include "bicg_state.hpp"
 #include "common.hpp"
 #include "persist_host.hpp"
 #include "persist_plan.hpp"
-
-struct BiDevState
-{
-    double norm_b;
-    double rel_tol;
-    double abs_tol;
-    double init_res;
-    double cur_res;
-    double alpha_stop;  // alpha of the iteration that stopped at the first check
-    int max_iters;
-    int n_prior;        // the solver control's nIters before the call
-    int iter;           // iterations completed
-    int done;
-    int stop_kind;      // 1: at the first check (x += alpha Mp pending), 2: at the second
-    int n_iters;
-    int converged;
-    int precond;
-    // Persistent iteration: grid-wide sums so far; 1 when a launch gave up
-    // waiting for another workgroup.
-    uint32_t epoch;
-    int failed;
-};
-
-namespace {
-
-__device__ __forceinline__ bool bi_finished(const BiDevState* st, double res, int it)
-{
-    const int n = (it == 0) ? st->n_prior : it;
-    return res <= st->rel_tol || res <= st->abs_tol * st->init_res || n >= st->max_iters;
-}
-
-}  // namespace
 
 // One launch: iterations from the state (x, r, r*, p, Mp = M p, <r*, r>) until
 // the device state says done (x complete, also after a stop at the first

@@ -89,13 +89,9 @@ __global__ __launch_bounds__(256) void bi_init_finalize(BiDevState* __restrict__
     }
 }
 
-// After a start from the x that a launch which gave up had left.
-__global__ void bi_recover(BiDevState* st, double init_res)
+__global__ void bi_recover_kernel(BiDevState* st, double init_res, int iter)
 {
-    if (threadIdx.x == 0) {
-        st->failed = 0;
-        st->init_res = init_res;
-    }
+    if (threadIdx.x == 0) bi_recover(*st, init_res, iter);
 }
 
 // partials of <a, b> (and, with c, of <c, d>).
@@ -510,7 +506,7 @@ clsparseStatus bicg_solve(cldenseVector* x, const clsparseCsrMatrix* A, const cl
         if (status == clsparseSuccess && hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess)
             status = clsparseInvalidKernelExecution;
     }
-    int printed = 0;
+    int printed = 0, iter = 0;  // iter: iterations of the launches that did not give up
     while (status == clsparseSuccess) {
         std::unique_lock<std::mutex> one(persist_mutex(control->device), std::defer_lock);
         if (persist) {
@@ -532,10 +528,11 @@ clsparseStatus bicg_solve(cldenseVector* x, const clsparseCsrMatrix* A, const cl
         if (hs->failed) {  // gave up waiting for a workgroup: from x again, in separate launches
             persist = false;
             CLS_TRY(start());
-            hipLaunchKernelGGL(bi_recover, dim3(1), dim3(64), 0, s, B.st, hs->init_res);
+            hipLaunchKernelGGL(bi_recover_kernel, dim3(1), dim3(64), 0, s, B.st, sc->initialResidual, iter);
             CLS_HIP_TRY(hipGetLastError());
             continue;
         }
+        iter = hs->iter;
         if (sc->printMode == VERBOSE) {
             // the reference prints after every completed iteration (L262-265)
             for (int k = printed; k < hs->iter; ++k) {

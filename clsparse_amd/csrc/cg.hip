@@ -769,13 +769,9 @@ clsparseStatus cg_setup(const clsparseCsrMatrix* A, const T* x, const T* b, size
     return clsparseSuccess;
 }
 
-// After a set-up from the x that a launch which gave up had left.
-__global__ void state_recover(CgDevState* st, double init_res)
+__global__ void state_recover(CgDevState* st, double init_res, int iter)
 {
-    if (threadIdx.x == 0) {
-        st->failed = 0;
-        st->init_res = init_res;
-    }
+    if (threadIdx.x == 0) cg_recover(*st, init_res, iter);
 }
 
 // The device-resident PCG loop on one system. x, b are T vectors of length n.
@@ -889,18 +885,19 @@ public:
     }
 
     // Runs chunks until the device state says done. `on_chunk` sees the host
-    // copy of the state after every chunk.
+    // copy of the state after every chunk. init_res: of the set-up.
     template <typename F>
-    clsparseStatus run(CgDevState* host_state, int max_run, F&& on_chunk)
+    clsparseStatus run(CgDevState* host_state, double init_res, int max_run, F&& on_chunk)
     {
-        for (;;) {
+        for (int iter = 0;;) {
             CLS_TRY(run_chunk(host_state, max_run));
             if (host_state->failed) {
                 CLS_TRY(cg_setup<T>(A_, x_, b_, n_, prec_, crit_, buf_, s_, ext_, false, nullptr));
-                hipLaunchKernelGGL(state_recover, dim3(1), dim3(64), 0, s_, buf_.st, host_state->init_res);
+                hipLaunchKernelGGL(state_recover, dim3(1), dim3(64), 0, s_, buf_.st, init_res, iter);
                 CLS_HIP_TRY(hipGetLastError());
                 continue;
             }
+            iter = host_state->iter;
             on_chunk(*host_state);
             if (host_state->done) break;
         }
@@ -1304,7 +1301,7 @@ clsparseStatus cg_solve(cldenseVector* x, const clsparseCsrMatrix* A, const clde
     int printed = 0;
     // VERBOSE prints every residual from the history ring: kChunk at a time.
     const int max_run = sc->printMode == VERBOSE ? kChunk : kMaxRun;
-    CLS_TRY(eng.run(hs, max_run, [&](const CgDevState& st) {
+    CLS_TRY(eng.run(hs, sc->initialResidual, max_run, [&](const CgDevState& st) {
         const int upto = st.done ? st.n_iters + 1 : st.iter;
         if (sc->printMode == VERBOSE) {
             for (int k = printed; k < upto; ++k) {
@@ -2025,6 +2022,9 @@ clsparseStatus reliable_solve(cldenseVector* x, const clsparseCsrMatrix* A, cons
             CLS_TRY(eng->run_chunk(hs, phase == kMain ? kMaxRun : kChunk, delta * res_at_replace, best_res));
             if (hs->failed) {  // a persistent launch gave up: from x again, in separate launches
                 bool over = false;
+                hs->iter = iter_at_chunk;
+                hipLaunchKernelGGL(state_recover, dim3(1), dim3(64), 0, s, buf.st, 0.0, iter_at_chunk);
+                CLS_HIP_TRY(hipGetLastError());
                 CLS_TRY(switch_to(eng, &over));
                 if (over) break;
                 continue;

@@ -1,8 +1,9 @@
 // Device state of one CG solve, shared by the launch-per-step iteration
-// (cg.hip) and the persistent one (cg_persist.hip).
+// (cg.hip) and the persistent ones (cg_persist_kernel.hpp, fsai_persist.hip).
+// Plain C++ (host and device): the host tests compile this header with g++.
 #pragma once
 
-#include "common.hpp"
+#include "persist_plan.hpp"
 
 namespace {
 
@@ -50,3 +51,20 @@ struct CgDevState
     double best_res;  // persistent learned-FSAI iteration: fsai_persist.hpp
     double hist[kHist];
 };
+
+// After a launch that gave up and a set-up from the x it left: the state of a
+// solve after `iter` iterations (those before that launch). Some workgroups may
+// have come to the launch's end all the same, with the sums of the one that gave
+// up: the state then says done, and x is theirs and older rows mixed.
+PP_HD inline void cg_recover(CgDevState& st, double init_res, int iter)
+{
+    st.failed = 0;
+    st.done = 0;
+    st.stop = 0;
+    st.converged = 0;
+    st.n_iters = 0;
+    st.pending = 0;
+    st.first = 1;
+    st.iter = iter;
+    st.init_res = init_res;
+}

@@ -14,7 +14,8 @@ unsigned long long persist_slot_empty();
 std::mutex& persist_mutex(int device);
 // Polls before a workgroup of a persistent kernel gives up waiting for another
 // (CLSPARSE_AMD_PERSIST_SPIN=<n>; default: seconds). The solve then goes on in
-// separate launches from the x it had before that launch.
+// separate launches from the x it had before that launch, with the rows of
+// workgroups that came to the launch's end as these have left them.
 int persist_spin_limit();
 // CLSPARSE_AMD_CG_PERSIST=0 keeps the launch-per-step iterations.
 bool persist_enabled();
