@@ -97,6 +97,10 @@ class clsparseAmdSolverStats(Structure):
                 ("loss_fsai", c_double), ("loss_jacobi", c_double)]
 
 
+class clsparseAmdSolverLaunches(Structure):
+    _fields_ = [("started", c_int32), ("refused", c_int32), ("gave_up", c_int32)]
+
+
 class clsparseAmdHostCsr(Structure):
     _fields_ = [("num_rows", c_uint32), ("num_cols", c_uint32), ("num_nonzeros", c_uint32),
                 ("row_pointer", POINTER(c_uint32)), ("col_indices", POINTER(c_uint32)),
@@ -159,6 +163,7 @@ _SIGS = {
                                                  c_uint32, POINTER(c_uint32)]),
     "clsparseAmdComputeRowBlocksHost": (c_uint64, [POINTER(c_uint32), c_uint32, POINTER(c_uint64)]),
     "clsparseAmdGetSolverStats": (c_int32, [_V, POINTER(clsparseAmdSolverStats)]),
+    "clsparseAmdGetSolverLaunches": (c_int32, [_V, POINTER(clsparseAmdSolverLaunches)]),
     "clsparseAmdDcsrcgMixed": (c_int32, [POINTER(cldenseVector), POINTER(clsparseCsrMatrix),
                                          POINTER(cldenseVector), _V, _V]),
     "clsparseAmdDcsrcgRefined": (c_int32, [POINTER(cldenseVector), POINTER(clsparseCsrMatrix),

@@ -305,6 +305,15 @@ extern "C" clsparseStatus clsparseSolverPrintMode(clSParseSolverControl solverCo
     return clsparseSuccess;
 }
 
+extern "C" clsparseStatus clsparseAmdGetSolverLaunches(clSParseSolverControl solverControl,
+                                                       clsparseAmdSolverLaunches* out)
+{
+    if (solverControl == nullptr) return clsparseInvalidSolverControlObject;
+    if (out == nullptr) return clsparseInvalidValue;
+    *out = solverControl->launches;
+    return clsparseSuccess;
+}
+
 extern "C" clsparseStatus clsparseAmdGetSolverStats(clSParseSolverControl solverControl,
                                                     clsparseAmdSolverStats* out)
 {

@@ -422,6 +422,7 @@ clsparseStatus bicg_solve(cldenseVector* x, const clsparseCsrMatrix* A, const cl
     CLS_HIP_TRY(hipStreamSynchronize(s));
     const double norm_b = hp->norm_b;
     sc->stats = clsparseAmdSolverStats{};
+    sc->launches = clsparseAmdSolverLaunches{};
     if (norm_b <= static_cast<double>(std::numeric_limits<T>::min())) {
         // x = b and zero tolerances (L75-83)
         sc->nIters = 0;
@@ -513,9 +514,11 @@ clsparseStatus bicg_solve(cldenseVector* x, const clsparseCsrMatrix* A, const cl
             one.lock();
             if (launch_bicg_persist<T>(pa, s) != clsparseSuccess) {  // nothing ran
                 (void)hipGetLastError();
+                ++sc->launches.refused;
                 persist = false;
                 continue;
             }
+            ++sc->launches.started;
         } else if (use_graph) {
             if (hipGraphLaunch(exec, s) != hipSuccess) status = clsparseInvalidKernelExecution;
         } else {
@@ -526,6 +529,7 @@ clsparseStatus bicg_solve(cldenseVector* x, const clsparseCsrMatrix* A, const cl
         CLS_HIP_TRY(hipMemcpyAsync(hs, B.st, sizeof(BiDevState), hipMemcpyDeviceToHost, s));
         CLS_HIP_TRY(hipStreamSynchronize(s));
         if (hs->failed) {  // gave up waiting for a workgroup: from x again, in separate launches
+            ++sc->launches.gave_up;
             persist = false;
             CLS_TRY(start());
             hipLaunchKernelGGL(bi_recover_kernel, dim3(1), dim3(64), 0, s, B.st, sc->initialResidual, iter);

@@ -789,9 +789,9 @@ public:
              CgBuffers<T>& buf, hipStream_t s, bool ext, const clsparseCsrMatrix* G = nullptr,
              const clsparseCsrMatrix* GT = nullptr, bool g_bf16 = false,
              const FsaiDia* dia = nullptr, const DiaMatrix<T>* adia = nullptr, T* r_alt = nullptr,
-             int num_cus = 0, int device = 0)
+             int num_cus = 0, int device = 0, clsparseAmdSolverLaunches* launches = nullptr)
         : A_(A), x_(x), b_(b), n_(n), prec_(prec), crit_(crit), buf_(buf), s_(s), ext_(ext),
-          g_(grid_for(n)), G_(G), GT_(GT), g_bf16_(g_bf16), r_alt_(r_alt), device_(device)
+          g_(grid_for(n)), G_(G), GT_(GT), g_bf16_(g_bf16), r_alt_(r_alt), device_(device), launches_(launches)
     {
         if (adia != nullptr && adia->vals != nullptr) adia_ = *adia;
         if (std::is_same_v<T, TX> && prec_ != kPrecFsai && adia_.vals != nullptr)
@@ -1014,12 +1014,17 @@ private:
         std::lock_guard<std::mutex> one(persist_mutex(device_));
         if (launch() != clsparseSuccess) {  // e.g. fewer CUs than the device has: nothing ran
             (void)hipGetLastError();
+            ++launches_->refused;
             persist_ = false;
             return clsparseSuccess;
         }
+        ++launches_->started;
         CLS_HIP_TRY(hipMemcpyAsync(host_state, buf_.st, sizeof(CgDevState), hipMemcpyDeviceToHost, s_));
         CLS_HIP_TRY(hipStreamSynchronize(s_));
-        if (host_state->failed) persist_ = false;
+        if (host_state->failed) {
+            ++launches_->gave_up;
+            persist_ = false;
+        }
         return clsparseSuccess;
     }
 
@@ -1193,6 +1198,7 @@ private:
     bool g_bf16_;
     T* r_alt_;
     int device_;
+    clsparseAmdSolverLaunches* launches_;  // of the solve
     PersistPlan plan_{};
     bool persist_ = false;      // whole chunks in one cooperative launch (cg_persist.hpp)
     bool fuse_gt_ = false;  // learned factor in diagonal storage: x / r update fused into G^T r
@@ -1245,6 +1251,7 @@ clsparseStatus cg_solve(cldenseVector* x, const clsparseCsrMatrix* A, const clde
         if (n > 0)
             CLS_HIP_TRY(hipMemcpyAsync(xp, bp, n * sizeof(T), hipMemcpyDeviceToDevice, s));
         sc->stats = clsparseAmdSolverStats{};
+        sc->launches = clsparseAmdSolverLaunches{};
         CLS_TRY(leave_solver_stream(control));
         return clsparseSuccess;
     }
@@ -1287,10 +1294,11 @@ clsparseStatus cg_solve(cldenseVector* x, const clsparseCsrMatrix* A, const clde
     if (a_ndiag && hp->dia_bad) a_ndiag = 0;
     if (a_ndiag) adia = DiaMatrix<T>{a_dia, a_ndiag, hp->dia_unsym == 0, a_off};
     CgEngine<T> eng(A, xp, bp, n, prec, kCritL1Ref, buf, s, control->extended_precision, nullptr, nullptr,
-                    false, nullptr, &adia, nullptr, control->num_cus, control->device);
+                    false, nullptr, &adia, nullptr, control->num_cus, control->device, &sc->launches);
 
     sc->initialResidual = hp->init_res;  // L127-129
     sc->stats = clsparseAmdSolverStats{};
+    sc->launches = clsparseAmdSolverLaunches{};
     if (sc->finished(sc->initialResidual)) {  // L134-138 (uses the stored nIters)
         sc->nIters = 0;
         sc->stats.l1_residual = sc->initialResidual;
@@ -1800,6 +1808,7 @@ clsparseStatus reliable_solve(cldenseVector* x, const clsparseCsrMatrix* A, cons
     CLS_HIP_TRY(hipStreamSynchronize(s));
     const double norm_b = hp->norm_b;
     sc->stats = clsparseAmdSolverStats{};
+    sc->launches = clsparseAmdSolverLaunches{};
     if (norm_b == 0) {
         sc->nIters = 0;
         if (n > 0) CLS_HIP_TRY(hipMemcpyAsync(xp, bp, n * sizeof(double), hipMemcpyDeviceToDevice, s));
@@ -1925,9 +1934,9 @@ clsparseStatus reliable_solve(cldenseVector* x, const clsparseCsrMatrix* A, cons
     // rI holds the inner right-hand side for each set-up only: the learned
     // factor's fused iteration may keep r in it between iterations.
     Engine eng_main(&AI, xe, rI, n, prec, kCritL2, buf, s, false, G, GT, g_bf16, have_dia ? &dia : nullptr,
-                    &adia, rI, control->num_cus, control->device);
+                    &adia, rI, control->num_cus, control->device, &sc->launches);
     Engine eng_jac(&AI, xe, rI, n, kPrecJacobi, kCritL2, buf, s, false, nullptr, nullptr, false, nullptr,
-                   &adia, nullptr, control->num_cus, control->device);
+                   &adia, nullptr, control->num_cus, control->device, &sc->launches);
     Engine* eng = &eng_main;
     // A pilot race already run for this factor decides without a new one
     // (the factor object forgets it when G changes).

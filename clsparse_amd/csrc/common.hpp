@@ -64,6 +64,7 @@ struct _solverControl
 
     // Extension state (no reference counterpart).
     clsparseAmdSolverStats stats{};
+    clsparseAmdSolverLaunches launches{};
 
     // finished / converged: solver-control.hpp L47-64, same evaluation order.
     bool converged(double residuum)

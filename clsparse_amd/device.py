@@ -12,7 +12,7 @@ import numpy as np
 import torch
 
 from . import (DIAGONAL, NOPRECOND, QUIET, ClsparseError, check, cldenseVector,
-               clsparseAmdSolverStats, clsparseCsrMatrix, clsparseScalar, load)
+               clsparseAmdSolverLaunches, clsparseAmdSolverStats, clsparseCsrMatrix, clsparseScalar, load)
 
 _TORCH = {np.float32: torch.float32, np.float64: torch.float64}
 
@@ -147,6 +147,11 @@ class SolverControl:
         st = clsparseAmdSolverStats()
         check("clsparseAmdGetSolverStats", load().clsparseAmdGetSolverStats(self.handle, byref(st)))
         return st
+
+    def launches(self) -> clsparseAmdSolverLaunches:
+        n = clsparseAmdSolverLaunches()
+        check("clsparseAmdGetSolverLaunches", load().clsparseAmdGetSolverLaunches(self.handle, byref(n)))
+        return n
 
     def set_params(self, precond, max_iters, rel_tol, abs_tol) -> None:
         check("clsparseSetSolverParams",

@@ -73,6 +73,20 @@ typedef struct clsparseAmdSolverStats_
 CLSPARSE_EXPORT clsparseStatus
     clsparseAmdGetSolverStats(clSParseSolverControl solverControl, clsparseAmdSolverStats* out);
 
+/* How the last solve ran the iterations of stencil systems that fit one
+ * cooperative launch: launches that started, launches that the device refused
+ * (nothing ran) and launches that gave up waiting for a workgroup. After a refusal
+ * or a give-up a solve goes on in separate launches. All 0: it used those alone. */
+typedef struct clsparseAmdSolverLaunches_
+{
+    cl_int started;
+    cl_int refused;
+    cl_int gave_up;
+} clsparseAmdSolverLaunches;
+
+CLSPARSE_EXPORT clsparseStatus
+    clsparseAmdGetSolverLaunches(clSParseSolverControl solverControl, clsparseAmdSolverLaunches* out);
+
 /* Mixed-precision Jacobi-PCG with FP64 residual replacement (no reference
  * counterpart). A, x and b are FP64. One CG run keeps A's values and the
  * vectors r, z, p, A p in FP32 and accumulates every dot product and norm in
