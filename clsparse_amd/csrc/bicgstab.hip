@@ -512,7 +512,7 @@ clsparseStatus bicg_solve(cldenseVector* x, const clsparseCsrMatrix* A, const cl
         std::unique_lock<std::mutex> one(persist_mutex(control->device), std::defer_lock);
         if (persist) {
             one.lock();
-            if (launch_bicg_persist<T>(pa, s) != clsparseSuccess) {  // nothing ran
+            if (persist_refused() || launch_bicg_persist<T>(pa, s) != clsparseSuccess) {  // nothing ran
                 (void)hipGetLastError();
                 ++sc->launches.refused;
                 persist = false;

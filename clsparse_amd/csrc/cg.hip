@@ -845,16 +845,18 @@ public:
     // persistent iteration runs several chunks in one launch, at most max_run
     // iterations, while the residual after each is above go_on; where a launch
     // gave up (host_state->failed) the caller starts again from x, in separate
-    // launches from then on, as does a device that refuses the launch.
+    // launches from then on. A device that refuses the launch has run nothing of
+    // it: the chunk runs in separate launches.
     // With the learned factor it also returns after a chunk that does not
     // halve the best residual, best to start with, of the chunks before
     // (host_state->best_res then).
     clsparseStatus run_chunk(CgDevState* host_state, int max_run = kChunk, double go_on = -1.0, double best = 0.0)
     {
         if (persist_) {
-            if (prec_ == kPrecFsai) CLS_TRY(run_persistent_fsai(host_state, max_run, go_on, best));
-            else CLS_TRY(run_persistent(host_state, max_run, go_on));
-            if (persist_ || host_state->failed) return clsparseSuccess;
+            bool refused = false;
+            if (prec_ == kPrecFsai) CLS_TRY(run_persistent_fsai(host_state, max_run, go_on, best, &refused));
+            else CLS_TRY(run_persistent(host_state, max_run, go_on, &refused));
+            if (!refused) return clsparseSuccess;
         }
         const bool use_graph = graphs_enabled();
         if (use_graph && exec_ == nullptr) {
@@ -949,7 +951,7 @@ public:
     }
 
 private:
-    clsparseStatus run_persistent(CgDevState* host_state, int max_run, double go_on)
+    clsparseStatus run_persistent(CgDevState* host_state, int max_run, double go_on, bool* refused)
     {
         if constexpr (std::is_same_v<T, TX>) {
             CgPersistArgs<T> a{};
@@ -972,12 +974,12 @@ private:
             a.max_run = max_run;
             a.go_on = go_on;
             a.spin_limit = persist_spin_limit();
-            return run_alone(host_state, [&] { return launch_cg_persist<T>(a, s_); });
+            return run_alone(host_state, refused, [&] { return launch_cg_persist<T>(a, s_); });
         }
         return clsparseInvalidValue;
     }
 
-    clsparseStatus run_persistent_fsai(CgDevState* host_state, int max_run, double go_on, double best)
+    clsparseStatus run_persistent_fsai(CgDevState* host_state, int max_run, double go_on, double best, bool* refused)
     {
         if constexpr (std::is_same_v<T, float> && std::is_same_v<TX, float>) {
             FsaiPersistArgs a{};
@@ -1001,7 +1003,7 @@ private:
             a.go_on = go_on;
             a.best = best;
             a.spin_limit = persist_spin_limit();
-            return run_alone(host_state, [&] { return launch_fsai_persist(a, s_); });
+            return run_alone(host_state, refused, [&] { return launch_fsai_persist(a, s_); });
         }
         return clsparseInvalidValue;
     }
@@ -1009,13 +1011,14 @@ private:
     // One persistent kernel per device at a time: two that shared the CUs
     // could each hold some the other waits for.
     template <typename F>
-    clsparseStatus run_alone(CgDevState* host_state, F&& launch)
+    clsparseStatus run_alone(CgDevState* host_state, bool* refused, F&& launch)
     {
         std::lock_guard<std::mutex> one(persist_mutex(device_));
-        if (launch() != clsparseSuccess) {  // e.g. fewer CUs than the device has: nothing ran
+        if (persist_refused() || launch() != clsparseSuccess) {  // e.g. fewer CUs than the device has: nothing ran
             (void)hipGetLastError();
             ++launches_->refused;
             persist_ = false;
+            *refused = true;  // (and host_state is not written)
             return clsparseSuccess;
         }
         ++launches_->started;

@@ -21,6 +21,12 @@ int persist_spin_limit()
     return n > 0 ? n : kSpinLimit;
 }
 
+bool persist_refused()
+{
+    const char* e = std::getenv("CLSPARSE_AMD_PERSIST_REFUSE");
+    return e && e[0] == '1';
+}
+
 bool persist_enabled()
 {
     const char* e = std::getenv("CLSPARSE_AMD_CG_PERSIST");

@@ -17,5 +17,8 @@ std::mutex& persist_mutex(int device);
 // separate launches from the x it had before that launch, with the rows of
 // workgroups that came to the launch's end as these have left them.
 int persist_spin_limit();
+// CLSPARSE_AMD_PERSIST_REFUSE=1 (for tests): every persistent launch is taken as
+// refused by the device.
+bool persist_refused();
 // CLSPARSE_AMD_CG_PERSIST=0 keeps the launch-per-step iterations.
 bool persist_enabled();
