@@ -852,7 +852,7 @@ public:
     // (host_state->best_res then).
     clsparseStatus run_chunk(CgDevState* host_state, int max_run = kChunk, double go_on = -1.0, double best = 0.0)
     {
-        if (persist_) {
+        if (persistent()) {
             bool refused = false;
             if (prec_ == kPrecFsai) CLS_TRY(run_persistent_fsai(host_state, max_run, go_on, best, &refused));
             else CLS_TRY(run_persistent(host_state, max_run, go_on, &refused));
@@ -917,7 +917,11 @@ public:
     }
     int prec() const { return prec_; }
     bool fused() const { return fused_; }
-    bool persistent_fsai() const { return persist_ && prec_ == kPrecFsai; }
+    // A launch of the solve that gave up, of this engine or of another one on the
+    // same buffers, leaves the slots with the sums it published and the count of
+    // its sums behind: no launch of either runs on them again.
+    bool persistent() const { return persist_ && launches_->gave_up == 0; }
+    bool persistent_fsai() const { return persistent() && prec_ == kPrecFsai; }
 
     // After a chunk that ran `ran` iterations: r back in buf_.r when the
     // fused learned-FSAI iteration left it in r_alt (an odd count).
@@ -1024,10 +1028,7 @@ private:
         ++launches_->started;
         CLS_HIP_TRY(hipMemcpyAsync(host_state, buf_.st, sizeof(CgDevState), hipMemcpyDeviceToHost, s_));
         CLS_HIP_TRY(hipStreamSynchronize(s_));
-        if (host_state->failed) {
-            ++launches_->gave_up;
-            persist_ = false;
-        }
+        if (host_state->failed) ++launches_->gave_up;
         return clsparseSuccess;
     }
 
