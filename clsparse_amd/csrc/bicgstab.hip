@@ -496,17 +496,21 @@ clsparseStatus bicg_solve(cldenseVector* x, const clsparseCsrMatrix* A, const cl
     }
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    const bool use_graph = !persist && graphs_enabled();
+    const bool use_graph = graphs_enabled();
     clsparseStatus status = clsparseSuccess;
-    if (use_graph) {
+    auto chunk = [&]() -> clsparseStatus {
+        for (int k = 0; k < kBiChunk; ++k) CLS_TRY(enqueue_bi_iteration<T>(A, adia, xp, B, n, g, k & 1, s, ext));
+        return clsparseSuccess;
+    };
+    auto capture = [&]() -> clsparseStatus {
         CLS_HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        for (int k = 0; k < kBiChunk && status == clsparseSuccess; ++k)
-            status = enqueue_bi_iteration<T>(A, adia, xp, B, n, g, k & 1, s, ext);
+        const clsparseStatus st = chunk();
         const hipError_t e = hipStreamEndCapture(s, &graph);
-        if (status == clsparseSuccess && e != hipSuccess) status = clsparseInvalidKernelExecution;
-        if (status == clsparseSuccess && hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess)
-            status = clsparseInvalidKernelExecution;
-    }
+        CLS_TRY(st);
+        if (e != hipSuccess || hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess)
+            return clsparseInvalidKernelExecution;
+        return clsparseSuccess;
+    };
     int printed = 0, iter = 0;  // iter: iterations of the launches that did not give up
     while (status == clsparseSuccess) {
         std::unique_lock<std::mutex> one(persist_mutex(control->device), std::defer_lock);
@@ -520,10 +524,10 @@ clsparseStatus bicg_solve(cldenseVector* x, const clsparseCsrMatrix* A, const cl
             }
             ++sc->launches.started;
         } else if (use_graph) {
-            if (hipGraphLaunch(exec, s) != hipSuccess) status = clsparseInvalidKernelExecution;
+            if (exec == nullptr) status = capture();
+            if (status == clsparseSuccess && hipGraphLaunch(exec, s) != hipSuccess) status = clsparseInvalidKernelExecution;
         } else {
-            for (int k = 0; k < kBiChunk && status == clsparseSuccess; ++k)
-                status = enqueue_bi_iteration<T>(A, adia, xp, B, n, g, k & 1, s, ext);
+            status = chunk();
         }
         if (status != clsparseSuccess) break;
         CLS_HIP_TRY(hipMemcpyAsync(hs, B.st, sizeof(BiDevState), hipMemcpyDeviceToHost, s));

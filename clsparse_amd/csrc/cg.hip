@@ -810,10 +810,11 @@ public:
         // 23.2 ms, clsparseScsrcg 13.6-13.7 against 14.1 ms, the same iterates).
         // Its buffer resources take K n sizeof(T) bytes in 32 bits; larger
         // systems keep the separate kernels (whose SpMV then takes flat loads).
-        fused_ = !persist_ && std::is_same_v<T, float> && prec_ != kPrecFsai && adia_.vals != nullptr && cg_fuse_enabled() &&
-                 dia_buf_fits(adia_.ndiag, n, sizeof(T));
+        can_fuse_ = std::is_same_v<T, float> && prec_ != kPrecFsai && adia_.vals != nullptr && cg_fuse_enabled() &&
+                    dia_buf_fits(adia_.ndiag, n, sizeof(T));
         // CLSPARSE_AMD_CG_FUSE=0 keeps the separate x / r update (the same iterates).
-        fuse_gt_ = !persist_ && prec_ == kPrecFsai && use_dia_ && r_alt_ != nullptr && cg_fuse_enabled();
+        can_fuse_gt_ = prec_ == kPrecFsai && use_dia_ && r_alt_ != nullptr && cg_fuse_enabled();
+        start_kernels();
     }
     ~CgEngine()
     {
@@ -830,6 +831,7 @@ public:
             if (!x_zero) return clsparseInvalidValue;  // the wide-x engine starts from a given residual
             CLS_TRY(cg_setup<T>(A_, nullptr, b_, n_, prec_, crit_, buf_, s_, ext_, true, nullptr));
         }
+        start_kernels();
         if (prec_ == kPrecFsai) {
             CLS_TRY(apply_fsai(buf_.part_rz[1], nullptr));
             hipLaunchKernelGGL((cast_kernel<T, T>), dim3(ew_grid(n_)), dim3(256), 0, s_, n_, buf_.z,
@@ -897,6 +899,7 @@ public:
                 CLS_TRY(cg_setup<T>(A_, x_, b_, n_, prec_, crit_, buf_, s_, ext_, false, nullptr));
                 hipLaunchKernelGGL(state_recover, dim3(1), dim3(64), 0, s_, buf_.st, init_res, iter);
                 CLS_HIP_TRY(hipGetLastError());
+                start_kernels();
                 continue;
             }
             iter = host_state->iter;
@@ -955,6 +958,15 @@ public:
     }
 
 private:
+    // The kernels of the iterations after a set-up. Those that fuse the p update or
+    // G^T r go on from their own state only, not from a persistent launch's.
+    void start_kernels()
+    {
+        fused_ = can_fuse_ && !persistent();
+        fuse_gt_ = can_fuse_gt_ && !persistent();
+        at_start_ = true;
+    }
+
     clsparseStatus run_persistent(CgDevState* host_state, int max_run, double go_on, bool* refused)
     {
         if constexpr (std::is_same_v<T, TX>) {
@@ -1022,9 +1034,11 @@ private:
             (void)hipGetLastError();
             ++launches_->refused;
             persist_ = false;
+            if (at_start_) start_kernels();
             *refused = true;  // (and host_state is not written)
             return clsparseSuccess;
         }
+        at_start_ = false;
         ++launches_->started;
         CLS_HIP_TRY(hipMemcpyAsync(host_state, buf_.st, sizeof(CgDevState), hipMemcpyDeviceToHost, s_));
         CLS_HIP_TRY(hipStreamSynchronize(s_));
@@ -1205,6 +1219,8 @@ private:
     clsparseAmdSolverLaunches* launches_;  // of the solve
     PersistPlan plan_{};
     bool persist_ = false;      // whole chunks in one cooperative launch (cg_persist.hpp)
+    bool can_fuse_ = false, can_fuse_gt_ = false;  // where no persistent launch runs
+    bool at_start_ = true;      // no persistent launch since the set-up
     bool fuse_gt_ = false;  // learned factor in diagonal storage: x / r update fused into G^T r
     bool use_dia_ = false;
     FsaiDia dia_{};

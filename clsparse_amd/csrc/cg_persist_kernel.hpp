@@ -332,6 +332,7 @@ clsparseStatus launch_cg_persist(CgPersistArgs<T> a, hipStream_t s)
     else if (a.plan.ndiag <= 5) e = launch_rows<5, T>(a, s);
     else if (a.plan.ndiag <= 7) e = launch_rows<7, T>(a, s);
     else if (a.plan.ndiag <= 9) e = launch_rows<9, T>(a, s);
-    CLS_HIP_TRY(e);
-    return clsparseSuccess;
+    // (refused, for instance while another process runs cooperative launches: the
+    // caller goes on without, and without a word)
+    return e == hipSuccess ? clsparseSuccess : clsparseInvalidKernelExecution;
 }

@@ -394,6 +394,7 @@ clsparseStatus launch_fsai_persist(FsaiPersistArgs a, hipStream_t s)
     case 9: e = launch_rows<9>(a, s); break;
     default: break;
     }
-    CLS_HIP_TRY(e);
-    return clsparseSuccess;
+    // (refused, for instance while another process runs cooperative launches: the
+    // caller goes on without, and without a word)
+    return e == hipSuccess ? clsparseSuccess : clsparseInvalidKernelExecution;
 }
