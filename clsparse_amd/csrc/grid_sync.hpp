@@ -23,8 +23,11 @@
 // the other workgroups of the XCD still use) is needed. Every wave waits for
 // its stores before its workgroup publishes.
 //
-// Every wait ends: after spin_limit polls (kSpinLimit: seconds) the call gives up
-// and returns false, and the kernel returns without a result.
+// Every wait ends: after spin_limit polls (kSpinLimit: at a round trip to memory
+// each about 0.1 s, several times the longest launch) the call gives up and returns
+// false, and the kernel returns without a result. A workgroup is late by so much
+// only where something else holds its CU, for which a solve in separate launches
+// need not wait.
 #pragma once
 
 #include "common.hpp"
@@ -41,7 +44,7 @@ constexpr uint32_t kSlotStride = 3 * kSlotSet + 544;       // words between copi
 constexpr size_t kSlotWords = size_t(kSlotReplicas) * kSlotStride;
 constexpr unsigned long long kSlotEmpty = 0x7FF8DEADBEEF0001ull;  // a NaN no arithmetic produces
 constexpr unsigned long long kSlotNan = 0x7FF8000000000000ull;
-constexpr int kSpinLimit = 1 << 23;
+constexpr int kSpinLimit = 1 << 17;
 
 struct GridShared
 {
