@@ -17,8 +17,9 @@
 // takes as few lanes as its bytes allow, also where V does not divide the
 // columns (81 entries a row times 13 FP32 columns: 16 one-column lanes per row
 // 52 us, 4 four-column lanes with four nonzeros each 36 us; one FP64 column
-// 68 -> 30 us), and rows past kLongRow entries are shared by the workgroup (a
-// power-law matrix with 75,000-entry rows times 13 FP64 columns: 7.5 ms -> 0.41).
+// 68 -> 30 us), rows far longer than the mean are shared by the slots of their wave,
+// and rows past kLongRow entries by the workgroup (a power-law matrix with
+// 75,000-entry rows times 13 FP64 columns: 7.5 ms -> 0.41).
 // Waves walk consecutive rows and workgroups are remapped so each XCD covers
 // one contiguous range of rows (neighbouring rows share B rows in its L2). Each
 // element of C is summed in an order fixed by the shapes, so results are
@@ -97,7 +98,7 @@ __device__ __forceinline__ void slot_sum(Cols<T, V>& sum, uint32_t beg, uint32_t
         if constexpr (Q > 1) {
             typedef uint32_t cvec __attribute__((ext_vector_type(Q), aligned(4)));
             typedef T tvec __attribute__((ext_vector_type(Q), aligned(sizeof(T))));
-            if (jj < end && jj + Q <= nnz) {
+            if (jj < end && nnz - jj >= Q) {
                 const cvec c4 = *reinterpret_cast<const cvec*>(ci + jj);
                 const tvec v4 = *reinterpret_cast<const tvec*>(v + jj);
 #pragma unroll
@@ -138,13 +139,30 @@ __device__ __forceinline__ void slot_sum(Cols<T, V>& sum, uint32_t beg, uint32_t
                 for (int k = 0; k < V; ++k) b8[u].e[k] = T(0);
                 if (colok && q + u < cnt) b8[u] = load_cols<T, V>(Bc + static_cast<size_t>(col) * ldb);
             }
+            // No branch around the products (b8 is 0 past cnt): 1024^2 rows of 3 entries
+            // near the diagonal times 32 FP64 columns 59 -> 53 us. Not so with four nonzeros a
+            // lane in wide slots, whose loads then all arrive before the first product: random
+            // rows of 200 times 16 FP64 columns 40 us with branches, 52 without.
+            constexpr bool kBranch = Q > 1 && W >= 8;
 #pragma unroll
-            for (int u = 0; u < kIn; ++u)
-                if (q + u < cnt)
+            for (int u = 0; u < kIn; ++u) {
+                if (kBranch && q + u >= cnt) continue;
+                const T a = q + u < cnt ? a8[u] : T(0);
 #pragma unroll
-                    for (int k = 0; k < V; ++k) sum.e[k] = fma(a8[u], b8[u].e[k], sum.e[k]);
+                for (int k = 0; k < V; ++k) sum.e[k] = fma(a, b8[u].e[k], sum.e[k]);
+            }
         }
     }
+}
+
+// The sum of a lane's columns over the slots of its wave, in every one of them.
+template <int W, typename T, int V>
+__device__ __forceinline__ void add_slots(Cols<T, V>& sum)
+{
+#pragma unroll
+    for (int d = W; d < 64; d *= 2)
+#pragma unroll
+        for (int k = 0; k < V; ++k) sum.e[k] += __shfl_xor(sum.e[k], d, 64);
 }
 
 // The lane's columns of one row of C: out = beta out + sum; only the columns
@@ -168,9 +186,12 @@ __device__ __forceinline__ void finish_cols(T* out, Cols<T, V> sum, T beta, uint
 
 // W lanes per row slot, V columns per lane, Q nonzeros per lane and trip.
 // RAGGED (V does not divide ncols, ncols >= V): the last group of a row starts
-// early and stores the columns that are its own.
+// early and stores the columns that are its own. Rows of more than wave_row entries
+// are taken by all slots of the wave. Eight waves per SIMD with one nonzero a lane,
+// four with four, are the most that the loads in flight leave registers for.
 template <typename T, int W, int V, int Q, bool RAGGED>
-__global__ __launch_bounds__(256) void csrmm_kernel(uint32_t num_rows, uint32_t ncols, uint32_t nnz,
+__global__ __launch_bounds__(256, Q == 1 ? 8 : 4) void csrmm_kernel(uint32_t num_rows, uint32_t ncols, uint32_t nnz,
+                                                    uint32_t wave_row,
                                                     const uint32_t* __restrict__ rp,
                                                     const uint32_t* __restrict__ ci,
                                                     const T* __restrict__ v, const T* __restrict__ B,
@@ -234,15 +255,41 @@ __global__ __launch_bounds__(256) void csrmm_kernel(uint32_t num_rows, uint32_t 
             }
             nlong += __popcll(bits);
         }
-        for (uint32_t c0 = 0; c0 < ncols; c0 += W * V) {
-            const uint32_t c = c0 + t * V;
-            const uint32_t cs = RAGGED ? min(c, ncols - V) : c;
-            Cols<T, V> sum;
+        // Rows far longer than the mean follow after the others, one by one, W Q
+        // nonzeros to each slot of the wave in turn (200,000 rows of 4 entries, every 50th
+        // of 300, times 13 FP32 columns: the wave waited 86 us for those slots; 37).
+        unsigned long long wave_rows = 0;
+        const uint32_t first_beg = beg, first_end = end;
+        uint32_t at = row, step = W * Q;
+        if constexpr (W < 64) {
+            const bool far = live && end - beg > wave_row;
+            wave_rows = __ballot(far && t == 0);
+            if (far) {
+                live = false;
+                end = beg;
+            }
+        }
+        for (bool shared = false;; shared = true) {
+            for (uint32_t c0 = 0; c0 < ncols; c0 += W * V) {
+                const uint32_t c = c0 + t * V;
+                const uint32_t cs = RAGGED ? min(c, ncols - V) : c;
+                Cols<T, V> sum;
 #pragma unroll
-            for (int k = 0; k < V; ++k) sum.e[k] = T(0);
-            if (alpha != T(0))
-                slot_sum<T, W, V, Q>(sum, beg, end, W * Q, nnz, ci, v, B + cs, ldb, alpha, c < ncols, t, base);
-            if (live && c < ncols) finish_cols<RAGGED, T, V>(C + static_cast<size_t>(row) * ldc + cs, sum, beta, c - cs);
+                for (int k = 0; k < V; ++k) sum.e[k] = T(0);
+                if (alpha != T(0))
+                    slot_sum<T, W, V, Q>(sum, beg, end, step, nnz, ci, v, B + cs, ldb, alpha, c < ncols, t, base);
+                if (shared) add_slots<W>(sum);
+                if (live && c < ncols)
+                    finish_cols<RAGGED, T, V>(C + static_cast<size_t>(at) * ldc + cs, sum, beta, c - cs);
+            }
+            if (wave_rows == 0) break;
+            const int owner = __builtin_ctzll(wave_rows);
+            wave_rows &= wave_rows - 1;
+            beg = __shfl(first_beg, owner, 64) + slot * (W * Q);
+            end = __shfl(first_end, owner, 64);
+            step = kSlots * W * Q;
+            at = row0 + static_cast<uint32_t>(owner) / W;
+            live = slot == 0;
         }
     }
     if (lane == 0) long_count[wv] = min(nlong, kLongList);
@@ -264,10 +311,7 @@ __global__ __launch_bounds__(256) void csrmm_kernel(uint32_t num_rows, uint32_t 
             if (alpha != T(0))
                 slot_sum<T, W, V, Q>(sum, mine, end, 4 * kSlots * W * Q, nnz, ci, v, B + cs, ldb, alpha, c < ncols, t,
                                      base);
-#pragma unroll
-            for (uint32_t d = W; d < 64; d *= 2)
-#pragma unroll
-                for (int k = 0; k < V; ++k) sum.e[k] += __shfl_xor(sum.e[k], static_cast<int>(d), 64);
+            add_slots<W>(sum);
             if (slot == 0)
 #pragma unroll
                 for (int k = 0; k < V; ++k) part[wv][t * V + k] = sum.e[k];
@@ -302,7 +346,9 @@ clsparseStatus launch_csrmm(int num_cus, hipStream_t s, uint32_t n, uint32_t nco
     const uint32_t want = (n + kRows - 1) / kRows;
     const uint32_t resident = std::max<uint32_t>(8u, static_cast<uint32_t>(per_cu * std::max(num_cus, 1)) / 8 * 8);
     const uint32_t grid = std::min<uint32_t>(resident, (want + 7) / 8 * 8);
-    hipLaunchKernelGGL((csrmm_kernel<T, W, V, Q, RAGGED>), dim3(grid), dim3(256), 0, s, n, ncols, nnz, rp, ci, v, B, ldb, C,
+    // Far longer than the mean: a row of eight times as many, and of sixteen trips.
+    const uint32_t wave_row = std::max<uint32_t>(16u * W * Q, 8 * (nnz / n));
+    hipLaunchKernelGGL((csrmm_kernel<T, W, V, Q, RAGGED>), dim3(grid), dim3(256), 0, s, n, ncols, nnz, wave_row, rp, ci, v, B, ldb, C,
                        ldc, pa, pb);
     CLS_HIP_TRY(hipGetLastError());
     return clsparseSuccess;
@@ -346,18 +392,34 @@ clsparseStatus launch_csrmm_rows(const clsparseCsrMatrix* A, uint32_t ncols, con
     const T* v = dev_ptr<T>(A->values, A->off_values);
     if (rp == nullptr) return clsparseInvalidMemObject;
     // V columns per lane, 16 bytes of them where there are as many; W lanes per
-    // row slot (a power of two >= the column groups, at most 64).
+    // row slot (a power of two >= the column groups, at most 64). A count that V
+    // does not divide takes one column a lane where the slots of all rows are fewer
+    // than 512 waves: each row is then one slot's chain of trips, and more lanes make
+    // it shorter (1,850 rows of 81 times 13 FP32 columns 10.5 -> 9.2 us).
     constexpr uint32_t kVec = 16 / sizeof(T);
-    const uint32_t V = ncols >= kVec ? kVec : (ncols >= 2 ? 2u : 1u);
-    const uint32_t groups = (ncols + V - 1) / V;
-    const uint32_t W = groups > 32 ? 64u : groups > 16 ? 32u : groups > 8 ? 16u : groups > 4 ? 8u
-                                     : groups > 2 ? 4u : groups > 1 ? 2u : 1u;
+    auto lanes = [](uint32_t groups) {
+        return groups > 32 ? 64u : groups > 16 ? 32u : groups > 8 ? 16u : groups > 4 ? 8u : groups > 2 ? 4u
+                                                                                   : groups > 1 ? 2u : 1u;
+    };
+    uint32_t V = ncols >= kVec ? kVec : (ncols >= 2 ? 2u : 1u);
+    uint32_t W = lanes((ncols + V - 1) / V);
+    if (ncols % V != 0 && static_cast<uint64_t>(n) * W < 512 * 64) {
+        V = 1;
+        W = lanes(ncols);
+    }
     const uint32_t nnz = A->num_nonzeros;
     // Four nonzeros per lane and trip for rows of several trips (FP64, 8 columns,
     // W = 4: 5 entries a row 11.5 us with one and 15.2 with four, 9 entries 16.8 and
-    // 19.5; 81 entries 31 and 26).
+    // 19.5; 81 entries 31 and 26). With W = 16 rows of three to eight trips only where the
+    // half of the waves that four leave a CU hold all slots, or many times as many
+    // would be needed: 18,500 rows of 81 (4,600 waves, twice around) times 64 FP32
+    // columns 21 us with one and 28 with four; 1,850 rows 11.5 and 10.0, 74,000 random
+    // rows 170 and 150.
     const bool ragged = ncols % V != 0;
-    const bool quads = nnz > 3 * static_cast<uint64_t>(n) * W;
+    const uint64_t waves = static_cast<uint64_t>(n) * W / 64;
+    const bool twice = W == 16 && nnz <= 8 * static_cast<uint64_t>(n) * W &&
+                       waves > 16 * static_cast<uint64_t>(num_cus) && waves <= 64 * static_cast<uint64_t>(num_cus);
+    const bool quads = nnz > 3 * static_cast<uint64_t>(n) * W && !twice;
 #define CLS_CSRMM(WW, VV, QQ, RR) \
     CLS_TRY((launch_csrmm<T, WW, VV, QQ, RR>(num_cus, s, n, ncols, nnz, rp, ci, v, Bp, ldb, Cp, ldc, pa, pb)))
 #define CLS_CSRMM_Q(WW, VV)                  \
@@ -385,7 +447,15 @@ clsparseStatus launch_csrmm_rows(const clsparseCsrMatrix* A, uint32_t ncols, con
         if (W == 1) CLS_CSRMM_Q(1, 2);
         else CLS_CSRMM_Q(2, 2);
     } else {
-        CLS_CSRMM_Q(1, 1);
+        switch (W) {
+        case 64: CLS_CSRMM_Q(64, 1); break;
+        case 32: CLS_CSRMM_Q(32, 1); break;
+        case 16: CLS_CSRMM_Q(16, 1); break;
+        case 8: CLS_CSRMM_Q(8, 1); break;
+        case 4: CLS_CSRMM_Q(4, 1); break;
+        case 2: CLS_CSRMM_Q(2, 1); break;
+        default: CLS_CSRMM_Q(1, 1); break;
+        }
     }
 #undef CLS_CSRMM_Q
 #undef CLS_CSRMM
