@@ -70,6 +70,31 @@ PP_HD inline bool persist_live_thread(const PersistPlan& p, uint32_t wg, uint32_
     return t < persist_live_threads(p, wg);
 }
 
+// Lines: the columns that a workgroup with `live` columns copies for each of its own
+// levels (each column's place there; below 0 they wrap): `side` ones on both sides of
+// its 512, and in the last column tile of a line the `side` ones past its end that
+// are not among those (rows of the next line, which diagonals that run across line
+// ends read). Only the rows below the workgroup's own ones (kLower: left), only those
+// above (kUpper), or both.
+enum Side : int { kBoth, kLower, kUpper };
+
+struct PersistColumns
+{
+    uint32_t left, right, past, live;
+    PP_HD uint32_t count() const { return left + right + past; }
+    PP_HD uint32_t operator()(uint32_t e) const
+    {
+        return e < left ? e - left : e < left + right ? kPersistThreads + e - left : live + e - left - right;
+    }
+};
+
+PP_HD inline PersistColumns persist_columns(const PersistPlan& p, Side side, uint32_t live)
+{
+    const uint32_t idle = kPersistThreads - live;
+    return {side != kUpper ? p.side : 0, side != kLower ? p.side : 0,
+            side != kLower ? (p.side < idle ? p.side : idle) : 0, live};
+}
+
 inline void persist_copy(PersistPlan* p, int64_t from, int64_t len, int64_t at)
 {
     if (len <= 0) return;

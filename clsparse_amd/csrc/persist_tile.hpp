@@ -51,7 +51,6 @@ __device__ __forceinline__ double stencil_term(T v, T x)
 // copy), `where` its first N entries of this thread. side: only the rows below
 // the workgroup's own ones (kLower), only those above (kUpper), or both.
 constexpr uint32_t kNoRow = 0xFFFFFFFFu;
-enum Side : int { kBoth, kLower, kUpper };
 
 __device__ __forceinline__ void fill_where(const PersistPlan& pl, uint32_t first, uint32_t e, uint32_t& row, uint32_t& at)
 {
@@ -121,10 +120,8 @@ __device__ __forceinline__ void fill_tile(const PersistPlan& pl, uint32_t first,
             }
         }
     } else {
-        // The levels before the first and after the last, `side` columns on
-        // both sides of every level, and in the last column tile of a line, of
-        // `live` columns, the `side` ones past its end (rows of the next line,
-        // which diagonals that run across line ends read). One column a thread,
+        // The levels before the first and after the last, and of every level the
+        // columns beside the workgroup's own (persist_columns). One column a thread,
         // M of its levels at a time: the slowest workgroup's memory latencies
         // hold up all others. The first of them together with the two whole
         // levels where the caller has the slots for it (BiCGStab 85 x 90 x 80
@@ -132,12 +129,8 @@ __device__ __forceinline__ void fill_tile(const PersistPlan& pl, uint32_t first,
         // FP32 rows has no registers for them: 15.9 -> 16.6).
         constexpr bool kTogether = N == line_slots<R>();
         constexpr int M = kTogether ? N - 2 : N < R ? N : R;
-        const uint32_t left = SIDE != kUpper ? pl.side : 0, right = SIDE != kLower ? pl.side : 0;
-        const uint32_t past = SIDE != kLower ? min(pl.side, kGridThreads - live) : 0;
-        const uint32_t columns = left + right + past;
-        auto column = [&](uint32_t e) {  // the left ones wrap below 0
-            return e < left ? e - left : e < left + right ? kGridThreads + e - left : live + e - left - right;
-        };
+        const PersistColumns column = persist_columns(pl, SIDE, live);
+        const uint32_t columns = column.count();
         const uint32_t c = column(tid);
         if (SIDE != kUpper) get(first - pl.line + tid, 0);
         if (SIDE != kLower) get(first + R * pl.line + tid, 1);
