@@ -1,5 +1,5 @@
 """SpMV with metadata on both sides of the sizes at which the way its entries are read
-changes (24, in FP64 64, and 256 MB of values and columns; with extended precision also rows shorter
+changes (24 and 192 MB of values and columns, in FP64 24, 64 and 128; with extended precision also rows shorter
 and longer than 12): the oracle's bars, and the same bits from two calls. Rows of 20 and
 30 with parts of other lengths, so that few blocks are row-wise."""
 import numpy as np
@@ -13,10 +13,11 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("ext", [False, True], ids=["plain", "extended"])
 @pytest.mark.parametrize("dtype,nnz", [(np.float64, 2_050_000), (np.float64, 2_150_000), (np.float32, 3_100_000),
                                        (np.float64, 5_500_000), (np.float64, 5_700_000),
-                                       (np.float32, 3_200_000), (np.float64, 22_300_000), (np.float64, 22_500_000)])
+                                       (np.float32, 3_200_000), (np.float64, 11_100_000), (np.float64, 11_250_000),
+                                       (np.float32, 25_100_000), (np.float32, 25_250_000)])
 def test_long_rows(dtype, nnz, ext):
     mb = nnz * (4 + np.dtype(dtype).itemsize) / 2 ** 20
-    assert min(abs(mb - 24), abs(mb - 64), abs(mb - 256)) < 2
+    assert min(abs(mb - k) for k in (24, 64, 128, 192)) < 2
     say(f"spmv with metadata, {mb:.0f} MB of entries, {np.dtype(dtype).name} ext={ext}")
     rng = np.random.default_rng(nnz)
     lengths = np.concatenate([np.full(nnz // 100, 20), np.full(3, 5000), np.full(7, 1500)])
