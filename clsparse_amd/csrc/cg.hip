@@ -1847,7 +1847,7 @@ clsparseStatus reliable_solve(cldenseVector* x, const clsparseCsrMatrix* A, cons
     // pilot end point.
     const size_t bytes = (kMixed ? align_up(nnz * sizeof(TI)) : 0) + align_up(n * sizeof(double)) +
                          align_up(n * (kIncr ? sizeof(TI) : sizeof(double))) +
-                         align_up(8 * sizeof(double)) + align_up(n * sizeof(TI)) +
+                         align_up(2 * sizeof(double)) + align_up(n * sizeof(TI)) +
                          CgBuffers<TI>::bytes(n) + (fsai ? 2 * align_up(n * sizeof(double)) : 0) +
                          (a_ndiag ? align_up(a_ndiag * n * sizeof(TI)) : 0);
     void* work = nullptr;
@@ -1857,7 +1857,7 @@ clsparseStatus reliable_solve(cldenseVector* x, const clsparseCsrMatrix* A, cons
     double* r64 = c.take<double>(n);
     TI* xd = kIncr ? c.take<TI>(n) : nullptr;              // mixed: increment since the last flush
     double* xsave = kIncr ? nullptr : c.take<double>(n);  // FP64 x: last replacement point
-    double* sc64 = c.take<double>(8);  // [2]=-1, [3]=+1
+    double* sc64 = c.take<double>(2);  // -1, +1
     TI* rI = c.take<TI>(n);            // TI start residual; FSAI temporary afterwards
     CgBuffers<TI> buf;
     buf.carve(c, n);
@@ -1873,7 +1873,7 @@ clsparseStatus reliable_solve(cldenseVector* x, const clsparseCsrMatrix* A, cons
     init.max_iters = sc->maxIters - 1;
     init.crit = kCritL2;
     hipLaunchKernelGGL((solver_prepare_kernel<TI, CgDevState>), dim3(ew_grid(persist_slot_words())),
-                       dim3(256), 0, s, init, buf.st, buf.one, buf.zero, sc64 + 2, buf.slots,
+                       dim3(256), 0, s, init, buf.st, buf.one, buf.zero, sc64, buf.slots,
                        static_cast<uint32_t>(persist_slot_words()), persist_slot_empty());
     CLS_HIP_TRY(hipGetLastError());
 
@@ -1927,7 +1927,7 @@ clsparseStatus reliable_solve(cldenseVector* x, const clsparseCsrMatrix* A, cons
     auto true_residual = [&](double* rel) -> clsparseStatus {
         hipLaunchKernelGGL((flush_and_copy<TI>), dim3(ew_grid(n)), dim3(256), 0, s, n, xp, xd, bp, r64);
         CLS_HIP_TRY(hipGetLastError());
-        CLS_TRY(launch_csrmv<double>(sc64 + 2, A, xp, sc64 + 3, r64, s, control->extended_precision,
+        CLS_TRY(launch_csrmv<double>(sc64, A, xp, sc64 + 1, r64, s, control->extended_precision,
                                      nullptr));
         CLS_TRY(launch_reduce<double, double>(RedOp::Sqr, r64, nullptr, n, &hp->res, true,
                                               control->red_partials, s));
