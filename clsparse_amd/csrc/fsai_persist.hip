@@ -11,7 +11,7 @@
 // owner forms it: a barrier between the r update and G^T r would cost 2 us.
 //
 // Per iteration against the launch-per-step kernels: 30 x 40 x 28 24.1 -> 13.2
-// us, 64^3 23.3 -> 13.6, 100 x 90 x 110 31.4 -> 22.2, 120^3 40.7 -> 33.6, 128^3
+// us, 64^3 23.3 -> 13.6, 100 x 90 x 110 31.4 -> 22.2, 120^3 40.7 -> 27.5, 128^3
 // 41.9 -> 28.4 (the solver's residual replacements included: 1-3 us). What is
 // left is three grid sums and three fills (store, barrier, load: 3 us each) and
 // with 16 rows the rest of A from memory.
@@ -319,8 +319,8 @@ __global__ __launch_bounds__(kGridThreads) void fsai_persist_kernel(FsaiPersistA
 
 // A stays in registers up to 8 rows per thread; with 16, three diagonals in LDS
 // where the tile leaves room for them, and of a plan by lines (whose kernel has
-// registers left) up to two in registers: 128^3 30.4 -> 28.4 us, 120^3 35.5 ->
-// 33.6.
+// registers left) up to two in registers: 128^3 30.4 -> 28.4 us. 120^3 gained as
+// much, 35.5 -> 33.6, before other changes took it to 27.5.
 constexpr int kRegRows = 8, kFsaiRegs = 2, kFsaiKept = 3;
 // With 32 rows the eight waves of a CU wait for memory that the 32 of the
 // launch-per-step kernels overlap: 160^3 72 us an iteration against 65.7.
